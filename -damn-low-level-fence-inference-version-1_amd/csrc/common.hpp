@@ -177,18 +177,37 @@ __device__ __forceinline__ float block_reduce(float v, Op op, float* scratch) {
     }
 }
 
-// Runtime wave count version (blockDim.x multiple of 64, at most 16 waves).
+// The values N <= 16 waves left in LDS (s 16-byte aligned), combined in wave
+// order.  N is a constant, so the reads are independent 128-bit ones with one
+// wait; a loop over the launch's wave count instead reads one float, waits
+// (~100 clocks) and combines, up to 15 times in a row, which was 0.3-0.6 us of
+// a one-row kernel.
+template <int N, class Op>
+__device__ __forceinline__ float fold_waves(const float* s, Op op) {
+    static_assert(N >= 1 && N <= 16, "one value per wave");
+    f4 v[(N + 3) / 4];
+#pragma unroll
+    for (int i = 0; i < (N + 3) / 4; ++i) v[i] = *reinterpret_cast<const f4*>(s + 4 * i);
+    float r = v[0].x;
+#pragma unroll
+    for (int i = 1; i < N; ++i) r = op(r, v[i / 4][i % 4]);
+    return r;
+}
+
+// Runtime wave count version (blockDim.x multiple of 64, at most 16 waves;
+// `scratch` holds 16 floats, 16-byte aligned).  Wave 0 also fills the slots
+// past the last wave, with what leaves the result's bits alone: -0 for a sum,
+// its own value for a maximum.
 template <class Op>
 __device__ __forceinline__ float block_reduce_dyn(float v, Op op, float* scratch) {
     v = wave_reduce(v, op);
     const int nwaves = blockDim.x / kWave;
     if (nwaves == 1) return v;
-    const int wave = threadIdx.x / kWave;
-    if ((threadIdx.x % kWave) == 0) scratch[wave] = v;
+    const int wave = threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    if (lane == 0 || (wave == 0 && lane >= nwaves && lane < 16))
+        scratch[wave + lane] = std::is_same<Op, OpAdd>::value && lane != 0 ? -0.0f : v;
     __syncthreads();
-    float r = scratch[0];
-    for (int i = 1; i < nwaves; ++i) r = op(r, scratch[i]);
-    return r;
+    return fold_waves<16>(scratch, op);
 }
 
 // ------------------------------------------------------------------- host

@@ -116,7 +116,7 @@ __global__ __launch_bounds__(1024) void q8_gather_rms_kernel(float* out, const u
                                                              int64_t vocab, const int32_t* ids,
                                                              int64_t tokens, int dim, const float* w,
                                                              float eps, int vpt) {
-    __shared__ float red[16];
+    __shared__ __align__(16) float red[16];
     const int T = blockDim.x;
     const int dim4 = dim >> 2;
     const int64_t rb = static_cast<int64_t>(dim / 32) * 34;

@@ -76,7 +76,7 @@ __global__ __launch_bounds__(1024) void head_ops_vec_kernel(const HeadArgs args,
     constexpr int HD = 8 * G;
     constexpr int HALF = 4 * G;
     __shared__ __align__(16) float cs[2 * HALF];  // cos[HALF] then sin[HALF]
-    __shared__ float red[16];
+    __shared__ __align__(16) float red[16];
     const int T = blockDim.x;
     const int U = (nq + nkv) * G;
 

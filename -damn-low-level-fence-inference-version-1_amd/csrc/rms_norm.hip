@@ -32,7 +32,7 @@ template <int MAXV, bool RES, bool OUT32, bool OUT16>
 __global__ __launch_bounds__(1024) void rms_rows_vec_kernel(
     float* out, uint16_t* out16, float* hid, const float* x, const float* res, const float* w,
     int64_t rows, int n, int vpt, float eps) {
-    __shared__ float red[kMaxWaves];
+    __shared__ __align__(16) float red[kMaxWaves];
     const int T = blockDim.x;
     const int n4 = n >> 2;
     f4 wv[MAXV];  // the weights: the same for every row, loaded once

@@ -48,8 +48,8 @@ __global__ __launch_bounds__(TPR == 0 ? 1024 : 256) void softmax_vec_kernel(
     constexpr int BLOCK = TPR == 0 ? 0 : 256;
     constexpr int RPB = TPR == 0 ? 1 : BLOCK / TPR;
     constexpr int WPR = TPR == 0 ? 0 : TPR / kWave;
-    __shared__ float red_max[16];
-    __shared__ float red_sum[16];
+    __shared__ __align__(16) float red_max[16];
+    __shared__ __align__(16) float red_sum[16];
     const int tpr = TPR == 0 ? static_cast<int>(blockDim.x) : TPR;
     const int lt = threadIdx.x % tpr;
     const int sub = threadIdx.x / tpr;
