@@ -135,6 +135,22 @@ __device__ __forceinline__ int row_scatter_index(int sl) {
     return idx;
 }
 
+// Lane rows (16 lanes) r = 0 .. 3 each hold one term of four sums v[0 .. 3]:
+// every lane of row r gets sum r, (row 0 + row 1) + (row 2 + row 3).  The
+// gfx950 swaps exchange half the rows of two registers in one instruction, so
+// four sums take three swaps and three adds (and no LDS round trip).
+__device__ __forceinline__ float row_sums4(float v0, float v1, float v2, float v3) {
+    const auto bits = [](float v) { return __builtin_bit_cast(uint32_t, v); };
+    const auto add = [](auto pair) {
+        const uint32_t lo = pair[0], hi = pair[1];
+        return __builtin_bit_cast(float, lo) + __builtin_bit_cast(float, hi);
+    };
+    // rows: v0 of 0 + 1, v1 of 0 + 1, v0 of 2 + 3, v1 of 2 + 3
+    const float a = add(__builtin_amdgcn_permlane16_swap(bits(v0), bits(v1), false, false));
+    const float b = add(__builtin_amdgcn_permlane16_swap(bits(v2), bits(v3), false, false));
+    return add(__builtin_amdgcn_permlane32_swap(bits(a), bits(b), false, false));
+}
+
 // Split partials in ws (16-byte aligned), n_q * splits * (128 + 2) floats:
 // the o rows [n_q][splits][128], then the (m, l) pairs [n_q][splits][2].
 constexpr int kHD = 128;
@@ -158,7 +174,8 @@ constexpr int kPolicyDevice = 16;
 // before any use) and lane s the (m, l) of split s.  M = max m_s, c_s =
 // 2^(m_s - M) (0 for an empty split), L = sum l_s c_s by a DPP reduction; each
 // lane adds c_b o_b over its splits in order, the four lane groups are added
-// as (sg0 + sg1) + (sg2 + sg3), and every lane returns the four dims' o / L.
+// as (sg0 + sg1) + (sg2 + sg3), and lane (sg, j) returns o / L of dim
+// 64 half + 4j + sg.
 // Shared by the merge kernel and the split kernel's last-arrival merge, so
 // both give the same bits.
 // A wave-uniform pointer as the compiler's uniform value (lane 0's copy), so
@@ -172,7 +189,7 @@ __device__ __forceinline__ float* uniform_ptr(const float* p) {
 
 // o_head and ml_head are wave-uniform.
 template <int POLICY>
-__device__ __forceinline__ f4 merge_head_half(const float* o_head, const float* ml_head, int splits, int half,
+__device__ __forceinline__ float merge_head_half(const float* o_head, const float* ml_head, int splits, int half,
                                               int lane) {
     const __amdgpu_buffer_rsrc_t ro =
         __builtin_amdgcn_make_buffer_rsrc(uniform_ptr(o_head), 0, splits * kHD * 4, kRsrcWord3);
@@ -206,22 +223,13 @@ __device__ __forceinline__ f4 merge_head_half(const float* o_head, const float* 
         acc.z = __builtin_fmaf(cb, ov[i].z, acc.z);
         acc.w = __builtin_fmaf(cb, ov[i].w, acc.w);
     });
-#pragma unroll
-    for (int m = 16; m <= 32; m *= 2) {
-        acc.x += __shfl_xor(acc.x, m, kWave);
-        acc.y += __shfl_xor(acc.y, m, kWave);
-        acc.z += __shfl_xor(acc.z, m, kWave);
-        acc.w += __shfl_xor(acc.w, m, kWave);
-    }
-    if (L == 0.0f) return f4{0.0f, 0.0f, 0.0f, 0.0f};
-    return f4{acc.x / L, acc.y / L, acc.z / L, acc.w / L};
+    const float sum = row_sums4(acc.x, acc.y, acc.z, acc.w);
+    return L == 0.0f ? 0.0f : sum / L;
 }
 
 // merge_head_half's outputs: lane (sg, j) writes dim 64 half + 4j + sg.
-__device__ __forceinline__ void write_head_half(float* out, uint16_t* out16, int h, int half, int lane, f4 r) {
-    const int sg = lane >> 4;
-    const float v = sg == 0 ? r.x : sg == 1 ? r.y : sg == 2 ? r.z : r.w;
-    const int64_t at = static_cast<int64_t>(h) * kHD + 64 * half + 4 * (lane & 15) + sg;
+__device__ __forceinline__ void write_head_half(float* out, uint16_t* out16, int h, int half, int lane, float v) {
+    const int64_t at = static_cast<int64_t>(h) * kHD + 64 * half + 4 * (lane & 15) + (lane >> 4);
     if (out) out[at] = v;
     if (out16) out16[at] = f32_to_f16_bits(v);
 }
@@ -243,6 +251,14 @@ __device__ __forceinline__ void write_head_half(float* out, uint16_t* out16, int
 // the row to the caches.  The first sub-chunk's K and V loads (the first
 // two sub-chunks' with FENCE_ATTN_KV_BUFS 2) are issued before the
 // prologue, which runs while they are in flight.
+// What bounds it: latency, link after link.  At 2,916 positions (46 splits x
+// 16 workgroups) the launch is ~1.6 us, q arrives 1.2 us after a workgroup
+// starts on an idle CU and up to 3.8 us after on one whose earlier workgroups
+// already asked for their rows, scores to outputs take ~1 us, the partials'
+// stores, the arrival and the merge ~2 us.  V's loads behind q's arrival and
+// the row sums in registers instead of LDS took the call from 8.01 to 7.63 us
+// (GPU time, Qwen3-4B's 32 x 8 heads); K behind q too: 8.3 us, four heads per
+// workgroup: 9.8 us.
 // ARRIVE (with !FINAL, at most kWave splits): no merge launch.  The partials
 // are written with device-coherent stores (agent-scope atomic stores, which
 // write through the XCD's L2); once they have completed, the workgroup bumps
@@ -270,7 +286,8 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(float* __restrict_
     static_assert(!QK || (kThreads >= 3 * kWave && kUnits <= 2 * kWave), "prologue lanes");
     static_assert(kSub == kWave, "one position of a sub-chunk per lane in (B)");
     __shared__ float sp[2][GT][kSub];      // scores of even / odd sub-chunks
-    __shared__ __align__(16) float xo[kPG][GT][HD];
+    constexpr int kWaves = kThreads / kWave;
+    __shared__ float xo[kWaves][GT][HD];   // each wave's sums of its position groups
     __shared__ __align__(16) float qcs[QK ? HD : 1];            // prologue: cos[HALF] then sin[HALF]
     __shared__ __align__(16) float qs[QK ? GT : 1][HD];         // prologue: the prepared q heads
     __shared__ __align__(16) uint16_t kvn[QK ? 2 : 1][HD];      // prologue: position pos's k, v (binary16)
@@ -342,18 +359,24 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(float* __restrict_
     // Clamped: a valid cached position (row 0 for an empty range); with ROPE
     // never row pos, which this launch is writing, unless pos is 0.
     const int t_fill = (t_begin < t_end && !(QK && t_begin == pos)) ? t_begin : 0;
-    auto load_kv = [&](int t0, auto slot) {
-        h8(&kr)[kPPG] = kbuf[decltype(slot)::value];
-        h8(&vr)[kPPG] = vbuf[decltype(slot)::value];
-        bool(&on)[kPPG] = onbuf[decltype(slot)::value];
+    auto load_rows = [&](int t0, const uint16_t* base, h8(&row)[kPPG], bool(&on)[kPPG]) {
 #pragma unroll
         for (int i = 0; i < kPPG; ++i) {
             const int t = t0 + pg + kPG * i;
             on[i] = t < t_end;
             const int64_t tc = (on[i] && !(QK && t == pos)) ? t : t_fill;
-            kr[i] = __builtin_nontemporal_load(reinterpret_cast<const h8*>(kbase + tc * kv_dim));
-            vr[i] = __builtin_nontemporal_load(reinterpret_cast<const h8*>(vbase + tc * kv_dim));
+            row[i] = __builtin_nontemporal_load(reinterpret_cast<const h8*>(base + tc * kv_dim));
         }
+    };
+    auto load_k = [&](int t0, auto slot) {
+        load_rows(t0, kbase, kbuf[decltype(slot)::value], onbuf[decltype(slot)::value]);
+    };
+    auto load_v = [&](int t0, auto slot) {
+        load_rows(t0, vbase, vbuf[decltype(slot)::value], onbuf[decltype(slot)::value]);
+    };
+    auto load_kv = [&](int t0, auto slot) {
+        load_k(t0, slot);
+        load_v(t0, slot);
     };
     auto process = [&](int t0, auto slot) {
         h8(&kr)[kPPG] = kbuf[decltype(slot)::value];
@@ -485,7 +508,11 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(float* __restrict_
     // Issued whether or not the range is empty (then clamped and unused), so
     // that every path reaches the prologue's waits with the same loads in
     // flight and they wait for the prologue's own loads only.
-    load_kv(t_begin, Slot0{});
+    // With the prologue, V follows once q is here: a CU holds several of these
+    // workgroups, and q of the later ones queues behind every row the earlier
+    // ones have asked for.  V is used two barriers later than K.
+    load_k(t_begin, Slot0{});
+    if constexpr (!QK) load_v(t_begin, Slot0{});
     if (NB == 2 && t_begin + kSub < t_end) load_kv(t_begin + kSub, Slot1{});
     if constexpr (QK) {
         const int i = iu, g = gu;
@@ -498,6 +525,7 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(float* __restrict_
             qcs[HALF + lane] = sn;
         }
         __syncthreads();  // qcs
+        load_v(t_begin, Slot0{});
         if (unit_wave) {
             rope_unit<ROPE, G>(a, b, qcs, i);
             if (!isk) {
@@ -545,22 +573,23 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(float* __restrict_
         }
     }
 
-    // Sum the position groups' outputs (they share the running maximum).
+    // Sum the position groups' outputs (they share the running maximum): the
+    // wave's four in registers, row r ending with dims 8 sl + 4 k + r, then
+    // the waves' through LDS.
 #pragma unroll
-    for (int g = 0; g < GT; ++g) {
-        f4 lo, hi;
-        lo.x = o[g][0], lo.y = o[g][1], lo.z = o[g][2], lo.w = o[g][3];
-        hi.x = o[g][4], hi.y = o[g][5], hi.z = o[g][6], hi.w = o[g][7];
-        *reinterpret_cast<f4*>(&xo[pg][g][8 * sl]) = lo;
-        *reinterpret_cast<f4*>(&xo[pg][g][8 * sl + 4]) = hi;
-    }
+    for (int g = 0; g < GT; ++g)
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            xo[wave][g][8 * sl + 4 * k + (lane >> 4)] =
+                row_sums4(o[g][4 * k], o[g][4 * k + 1], o[g][4 * k + 2], o[g][4 * k + 3]);
     __syncthreads();
     // thread (g, d): one output element of one head
     for (int e = threadIdx.x; e < GT * HD; e += kThreads) {
         const int g = e / HD, d = e % HD;
         if (g >= ng) continue;
-        float acc = 0.0f;
-        for (int k = 0; k < kPG; ++k) acc += xo[k][g][d];
+        float acc = xo[0][g][d];
+#pragma unroll
+        for (int k = 1; k < kWaves; ++k) acc += xo[k][g][d];
         float l = hl[0], mg = hm[0];
 #pragma unroll
         for (int k = 1; k < GT; ++k) {
@@ -612,8 +641,8 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(float* __restrict_
         const int splits = static_cast<int>(gridDim.y);
         for (int e = wave; e < 2 * ng; e += kThreads / kWave) {
             const int h = h0 + e / 2;
-            const f4 r = merge_head_half<kPolicyDevice>(ws + partial_o_at(h, splits, 0),
-                                                        ws + partial_ml_at(n_q, h, splits, 0), splits, e % 2, lane);
+            const float r = merge_head_half<kPolicyDevice>(ws + partial_o_at(h, splits, 0),
+                                                           ws + partial_ml_at(n_q, h, splits, 0), splits, e % 2, lane);
             write_head_half(out, out16, h, e % 2, lane, r);
         }
     }
