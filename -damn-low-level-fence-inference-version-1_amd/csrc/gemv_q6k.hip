@@ -121,11 +121,11 @@ static_assert(FENCE_GEMV_Q6K_PAIRW == 0 || FENCE_GEMV_Q6K_PAIRW == 4 || FENCE_GE
 // computed (as XW launches do) in the one-wave launches with the RMSNorm
 // prologue (q/k/v) -- PF_NORM -- and in launches of several waves per row
 // (down) -- PF_SPLIT; 0: each group after the previous one.  Same results.
-// Measured as above: 1,693 us per token with PF_NORM against 1,685-1,687
-// without (97 VGPRs: 4 waves per SIMD instead of 5), 1,681-1,682 with
-// PF_SPLIT (within the spread of the session's runs).
+// PF_NORM: q/k/v of Qwen3-4B (6144 x 2560) 6.65 us without, 6.28 with, GPU
+// time (two 8-wave workgroups per CU either way, half of which take a second
+// group).  PF_SPLIT: decode steps within the spread of the runs.
 #ifndef FENCE_GEMV_Q6K_PF_NORM
-#define FENCE_GEMV_Q6K_PF_NORM 0
+#define FENCE_GEMV_Q6K_PF_NORM 1
 #endif
 #ifndef FENCE_GEMV_Q6K_PF_SPLIT
 #define FENCE_GEMV_Q6K_PF_SPLIT 0
@@ -303,7 +303,8 @@ __host__ __device__ constexpr int q6_wpr(int nb) {
 }
 __host__ __device__ constexpr int q6_passes(int nb) { return (nb + 4 * q6_wpr(nb) - 1) / (4 * q6_wpr(nb)); }
 
-// The lane's x pairs of every pass (binary16 zeros for a masked block).
+// The lane's x pairs of every pass (a masked block's are some block's: its
+// value is dropped where the passes are added).
 // Loads only: load_x_bias then forms the column biases, so loads issued in
 // between stay in flight while the biases wait for x.
 template <int PASSES>
@@ -326,8 +327,8 @@ __device__ __forceinline__ void load_x_pairs(uint32_t (&xh)[PASSES][8], const ui
                 lo = x16[e] | (static_cast<uint32_t>(x16[e + 1]) << 16);
                 hi = x16[e + 2] | (static_cast<uint32_t>(x16[e + 3]) << 16);
             }
-            xh[p][2 * c] = on ? lo : 0u;  // binary16 zeros: a masked block adds 0
-            xh[p][2 * c + 1] = on ? hi : 0u;
+            xh[p][2 * c] = lo;
+            xh[p][2 * c + 1] = hi;
         }
     }
 }
@@ -447,10 +448,10 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gem
     // NORM: binary16 x of the longest row this shape takes (nb <= 4 * PASSES * WPR)
     constexpr int kStageBytes = NW * kBufBytes;
     constexpr int kNormXBytes = 2 * 1024 * PASSES * WPR;
-    constexpr int kLdsBytes = NORM && kNormXBytes > kStageBytes ? kNormXBytes : kStageBytes;
+    constexpr int kLdsBytes = kStageBytes + (NORM ? kNormXBytes : 0);
     __shared__ __align__(16) uint8_t lds[kLdsBytes];
     __shared__ float red[NW];
-    __shared__ float nred[NORM ? 16 : 1];  // the row norm's wave sums (T <= 1024)
+    __shared__ __align__(16) float nred[NORM ? 16 : 1];  // the row norm's wave sums (T <= 1024)
     __shared__ float xr[XW ? NW : 1][XW ? PASSES : 1][kWave];  // XW: each pass's lane values
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));  // wave-uniform
@@ -473,12 +474,10 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gem
     float kb[PASSES][4];
     if constexpr (!NORM) load_x_pairs<PASSES>(xh, x16, b0, b1, bslot, h, j);  // biases once the first group is out
 
-    // NORM, first half: the row's loads, issued before the first group's
-    // blocks.  Wave w holds the row norm's waves w, w + NW, ... (vw < T / 64);
+    // NORM, first half: the row's loads.  Wave w holds the row norm's waves w, w + NW, ... (vw < T / 64);
     // a slot past the row holds zeros, as in the norm kernel.
     // Every load is unconditional (clamped slots, and hidden again in place of
-    // an absent residual), so all are in flight together and none waits for
-    // the blocks issued after them.
+    // an absent residual), so all are in flight together.
     static_assert(NORM == 0 || (VW >= 1 && VW * NW <= 16 + NW - 1), "VW: 1 .. ceil(16 / NW) slots");
     constexpr int kVW = NORM ? VW : 1;
     constexpr int kVpt = NORM ? NORM : 1;
@@ -548,17 +547,15 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gem
     };
     u4 ch[kChunkSlots];
     if constexpr (NORM != 0) {
-        // Second half, while the first group's blocks are in flight (the loop
-        // below does not load them again): the norm kernel's reduction, x into
-        // LDS, then each lane's x values.
-        {
-            int64_t o, lr, a0;
-            int m, nch;
-            uint32_t delta;
-            row_of(blockIdx.x, &o, &m, &lr);
-            seg_of(lr, &a0, &nch, &delta);
-            load_seg(job.W[m], a0, nch, ch);
-        }
+        // Second half: the norm kernel's reduction, x into LDS of its own (so
+        // that no barrier stands between a wave's x and its first staged
+        // blocks), then each lane's x values.  The first group's blocks are
+        // asked for once the row is here (the loop below does not load them
+        // again): asked for before, they delayed the row of the CU's second
+        // workgroup by 1-2 us, and nothing starts without it.  With the wave
+        // sums read at once (fold_waves) and the prefetch above, q/k/v of
+        // Qwen3-4B went from 7.0 to 6.3 us: 0.2 the order, 0.1 the barrier
+        // and the sums, 0.4 the prefetch.
         // h = hid (+ res), zero past the row; workgroup 0 stores it; then
         // each slot keeps only w * h, the first product of the norm's output
         const int nvw = rin.T / kWave;
@@ -584,17 +581,28 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gem
                 ss += kVpt > 1 ? dot4(nh[i][kVpt - 1]) : 0.0f;
                 ss = wave_reduce(ss, OpAdd{});
                 if (lane == 0) nred[vw] = ss;
+            } else if (vw < 16) {  // fold_waves reads it: +0 keeps the sum
+                if (lane == 0) nred[vw] = 0.0f;
             }
         }
 #pragma unroll
         for (int i = 0; i < kVW; ++i)
 #pragma unroll
             for (int jj = 0; jj < kVpt; ++jj) nw[i][jj] = nw[i][jj] * nh[i][jj];
+        __builtin_amdgcn_sched_barrier(0);
+        {
+            int64_t o, lr, a0;
+            int m, nch;
+            uint32_t delta;
+            row_of(blockIdx.x, &o, &m, &lr);
+            seg_of(lr, &a0, &nch, &delta);
+            load_seg(job.W[m], a0, nch, ch);
+        }
+        __builtin_amdgcn_sched_barrier(0);
         __syncthreads();
-        float tot = nred[0];
-        for (int v = 1; v < nvw; ++v) tot += nred[v];
+        const float tot = fold_waves<(kVW * NW < 16 ? kVW * NW : 16)>(nred, OpAdd{});
         const float rs = rsqrtf(tot / static_cast<float>(nb * 256) + rin.eps);
-        uint16_t* xs = reinterpret_cast<uint16_t*>(lds);
+        uint16_t* xs = reinterpret_cast<uint16_t*>(lds + kStageBytes);
 #pragma unroll
         for (int i = 0; i < kVW; ++i) {
 #pragma unroll
@@ -609,7 +617,6 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gem
         }
         __syncthreads();
         load_x<PASSES>(xh, kb, xs, b0, b1, bslot, h, j);
-        __syncthreads();  // lds holds staged blocks from here on
     }
     // One row group; LOADED: its blocks are already in ch (the NORM
     // prologue's first group), so the loop itself loads unconditionally.
@@ -777,9 +784,9 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(FENC
     constexpr uint32_t kPassBytes = 4 * kBlockBytes;
     constexpr int kStageBytes = NW * 2 * kBufBytes;
     constexpr int kNormXBytes = 2 * 1024 * PASSES;
-    constexpr int kLdsBytes = NORM && kNormXBytes > kStageBytes ? kNormXBytes : kStageBytes;
+    constexpr int kLdsBytes = kStageBytes + (NORM ? kNormXBytes : 0);
     __shared__ __align__(16) uint8_t lds[kLdsBytes];
-    __shared__ float nred[NORM ? 16 : 1];
+    __shared__ __align__(16) float nred[NORM ? 16 : 1];
     const int lane = threadIdx.x & (kWave - 1);
     const int wid = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x / kWave));
     uint8_t* bufg = lds + wid * (2 * kBufBytes);
@@ -935,6 +942,8 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(FENC
                 ss += kVpt > 1 ? dot4(nh[i][kVpt - 1]) : 0.0f;
                 ss = wave_reduce(ss, OpAdd{});
                 if (lane == 0) nred[vw] = ss;
+            } else if (vw < 16) {  // fold_waves reads it: +0 keeps the sum
+                if (lane == 0) nred[vw] = 0.0f;
             }
         }
 #pragma unroll
@@ -942,10 +951,9 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(FENC
 #pragma unroll
             for (int jj = 0; jj < kVpt; ++jj) nw[i][jj] = nw[i][jj] * nh[i][jj];
         __syncthreads();
-        float tot = nred[0];
-        for (int v = 1; v < nvw; ++v) tot += nred[v];
+        const float tot = fold_waves<(kVW * NW < 16 ? kVW * NW : 16)>(nred, OpAdd{});
         const float rs = rsqrtf(tot / static_cast<float>(nb * 256) + rin.eps);
-        uint16_t* xs = reinterpret_cast<uint16_t*>(lds);
+        uint16_t* xs = reinterpret_cast<uint16_t*>(lds + kStageBytes);
 #pragma unroll
         for (int i = 0; i < kVW; ++i) {
 #pragma unroll
@@ -961,7 +969,6 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(FENC
         __syncthreads();
         load_x<PASSES>(xh, kb, xs, b0, b1, bslot, h, j);
         if constexpr (MERGE) load_x<1>(xm, km, xs, b0m, b1, bslot, h, j);
-        __syncthreads();  // lds holds staged rows from here on
     }
     for (int64_t o = o0; o < n_out; o += waves) {  // wave-uniform
         int64_t a0;
