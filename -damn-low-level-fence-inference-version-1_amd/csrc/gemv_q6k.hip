@@ -393,7 +393,7 @@ __device__ __forceinline__ int mat_of(const Q6Job& job, int64_t r, int64_t* lr) 
     return m;
 }
 
-// Waves of a staged workgroup: 4; 8 for a gate/up pair whose rows take four
+// Waves of a staged workgroup: 4; 8 where x comes through LDS (XL below); 8 for a gate/up pair whose rows take four
 // waves each; 8 for a launch that normalises its input row in the prologue
 // with one wave per row (every workgroup computes the row norm, so wider
 // workgroups compute it fewer times per CU).  Measured on MI355X: two 8-wave
@@ -405,8 +405,8 @@ __device__ __forceinline__ int mat_of(const Q6Job& job, int64_t r, int64_t* lr) 
 // Qwen3-4B decode steps 1,718 -> 1,710 us per token against six 4-wave ones
 // (bench.py --decode-only, interleaved runs).  A row's arithmetic does not
 // depend on the workgroup, so every result is the same.
-template <int WPR, bool PAIR, int NORM = 0>
-constexpr int staged_waves() { return NORM && WPR == 1 ? 8 : (PAIR && WPR == 4 ? 8 : 4); }
+template <int WPR, bool PAIR, int NORM = 0, bool XL = false>
+constexpr int staged_waves() { return XL || (NORM && WPR == 1) ? 8 : (PAIR && WPR == 4 ? 8 : 4); }
 
 // Staged kernel.  WPR waves per row (1, 2 or 4), each over at most 4 * PASSES
 // <= 16 blocks.  LDS: one buffer of kSegBytes per wave + red[].  A workgroup
@@ -430,14 +430,24 @@ constexpr int staged_waves() { return NORM && WPR == 1 ? 8 : (PAIR && WPR == 4 ?
 // costs its loads, masks and reductions whether or not it is used).
 // CLOCK: the instrumented copy (FENCE_WAVE_CLOCK builds launch it on the grid
 // the plain kernel gets); every product launch has CLOCK = false.
-template <int PASSES, int WPR, bool PAIR, bool MULTI, int NORM, bool XW = false, bool CLOCK = false, int VW = 0>
-__global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gemv_q6k_staged_kernel(
+// XL (16-byte aligned x, rows on four waves of at most three passes): x comes
+// through LDS once per 8-wave workgroup.  A wave that loads its own x reads 2
+// KB a pass for 840 bytes of weights and visits one or two rows, so over the
+// six 4-wave workgroups of a CU x was more of its traffic than W.  Same bits.
+// Measured, GPU time: down 2560 x 9728 7.88 -> 7.44 us, o 2560 x 4096 4.39 ->
+// 4.32; with four passes (rows of 49-64 blocks) x takes 32 KB and only 16
+// waves fit a CU instead of 24: 4096 x 14336 13.3 -> 13.7, so those keep a
+// wave's own loads.
+template <int PASSES, int WPR, bool PAIR, bool MULTI, int NORM, bool XW = false, bool CLOCK = false, int VW = 0,
+          bool XL = false>
+__global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM, XL>())) void gemv_q6k_staged_kernel(
     const Q6Job job, const uint16_t* __restrict__ x16, int nb, const RmsIn rin) {
     static_assert(!XW || (PASSES * WPR == 4 && !PAIR && NORM == 0), "XW: four passes, plain rows");
     // prefetch the next row group: XW launches, and where the switches below ask
     constexpr bool PF = XW || (FENCE_GEMV_Q6K_PF_NORM && NORM != 0 && WPR == 1 && !PAIR) ||
                         (FENCE_GEMV_Q6K_PF_SPLIT && NORM == 0 && WPR > 1 && !PAIR);
-    constexpr int NW = staged_waves<WPR, PAIR, NORM>();
+    static_assert(!XL || (NORM == 0 && !PAIR && WPR == 4 && PASSES <= 3), "XL: plain rows of four waves");
+    constexpr int NW = staged_waves<WPR, PAIR, NORM, XL>();
     constexpr int kSegBytes = 4 * PASSES * kBlockBytes + 32;  // + alignment slack
     constexpr int kBufBytes = (kSegBytes + 15) / 16 * 16;
     constexpr int kChunkSlots = (kSegBytes / 16 + kWave - 1) / kWave;
@@ -448,7 +458,9 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gem
     // NORM: binary16 x of the longest row this shape takes (nb <= 4 * PASSES * WPR)
     constexpr int kStageBytes = NW * kBufBytes;
     constexpr int kNormXBytes = 2 * 1024 * PASSES * WPR;
-    constexpr int kLdsBytes = kStageBytes + (NORM ? kNormXBytes : 0);
+    constexpr int kXSlots = XL ? kNormXBytes / 16 / (kWave * NW) : 1;  // XL: x's 16-byte chunks per lane
+    static_assert(!XL || kXSlots * 16 * kWave * NW == kNormXBytes, "XL: whole chunks per lane");
+    constexpr int kLdsBytes = kStageBytes + (NORM || XL ? kNormXBytes : 0);
     __shared__ __align__(16) uint8_t lds[kLdsBytes];
     __shared__ float red[NW];
     __shared__ __align__(16) float nred[NORM ? 16 : 1];  // the row norm's wave sums (T <= 1024)
@@ -472,7 +484,16 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gem
 
     uint32_t xh[PASSES][8];
     float kb[PASSES][4];
-    if constexpr (!NORM) load_x_pairs<PASSES>(xh, x16, b0, b1, bslot, h, j);  // biases once the first group is out
+    u4 xc[kXSlots];
+    if constexpr (XL) {
+#pragma unroll
+        for (int k = 0; k < kXSlots; ++k) {
+            const int i = static_cast<int>(threadIdx.x) + kWave * NW * k;
+            xc[k] = reinterpret_cast<const u4*>(x16)[i < 32 * nb ? i : 0];  // past x: any of it, read by no lane
+        }
+    } else if constexpr (!NORM) {
+        load_x_pairs<PASSES>(xh, x16, b0, b1, bslot, h, j);  // biases once the first group is out
+    }
 
     // NORM, first half: the row's loads.  Wave w holds the row norm's waves w, w + NW, ... (vw < T / 64);
     // a slot past the row holds zeros, as in the norm kernel.
@@ -740,7 +761,15 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM>())) void gem
         seg_of(lr, &a0, &nch, &delta);
         load_seg(job.W[m], a0, nch, ch);
         __builtin_amdgcn_sched_barrier(0);
-        load_x_bias<PASSES>(xh, kb);
+        if constexpr (XL) {
+            uint16_t* xs = reinterpret_cast<uint16_t*>(lds + kStageBytes);
+#pragma unroll
+            for (int k = 0; k < kXSlots; ++k) reinterpret_cast<u4*>(xs)[threadIdx.x + kWave * NW * k] = xc[k];
+            __syncthreads();
+            load_x<PASSES>(xh, kb, xs, b0, b1, bslot, h, j);
+        } else {
+            load_x_bias<PASSES>(xh, kb);
+        }
     }
     if constexpr (PF) {  // every later group's chunks a group ahead
         for (int64_t g = blockIdx.x; g * kOutPerGroup < n_out; g += gridDim.x) run_group(g, std::true_type{});
@@ -1111,7 +1140,8 @@ int launch_grid_as(OccKernel occ_kernel, Kernel kernel, int threads, std::atomic
         if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, occ_kernel, threads, 0);
             e != hipSuccess)
             return hip_status(e);
-        if (FENCE_GEMV_Q6K_WG_PER_CU > 0 && per_cu > FENCE_GEMV_Q6K_WG_PER_CU) per_cu = FENCE_GEMV_Q6K_WG_PER_CU;
+        const int cap = FENCE_GEMV_Q6K_WG_PER_CU * 4 * kWave / threads;  // in waves: of 4-wave workgroups
+        if (FENCE_GEMV_Q6K_WG_PER_CU > 0 && per_cu > cap) per_cu = cap;
         g = cus * (per_cu > 0 ? per_cu : 1);
         cache[dev].store(g, std::memory_order_relaxed);
     }
@@ -1131,19 +1161,23 @@ int launch_grid(Kernel kernel, int threads, std::atomic<int>* cache, int64_t gro
     return launch_grid_as(kernel, kernel, threads, cache, groups, s, args...);
 }
 
-template <int PASSES, int WPR, bool PAIR, bool MULTI, int NORM, bool XW, int VW>
+template <int PASSES, int WPR, bool PAIR, bool MULTI, int NORM, bool XW, int VW, bool XL = false>
 int launch_staged_vw(const Q6Job& job, int64_t n_out, const uint16_t* x, int nb, const RmsIn& rin, hipStream_t s) {
     static std::atomic<int> cache[64];
-    constexpr int nw = staged_waves<WPR, PAIR, NORM>();
+    constexpr int nw = staged_waves<WPR, PAIR, NORM, XL>();
     constexpr int out_per_group = PAIR ? nw / WPR / 2 : nw / WPR;
-    return launch_grid_as(gemv_q6k_staged_kernel<PASSES, WPR, PAIR, MULTI, NORM, XW, false, VW>,
-                          gemv_q6k_staged_kernel<PASSES, WPR, PAIR, MULTI, NORM, XW, FENCE_WAVE_CLOCK != 0, VW>,
+    return launch_grid_as(gemv_q6k_staged_kernel<PASSES, WPR, PAIR, MULTI, NORM, XW, false, VW, XL>,
+                          gemv_q6k_staged_kernel<PASSES, WPR, PAIR, MULTI, NORM, XW, FENCE_WAVE_CLOCK != 0, VW, XL>,
                           kWave * nw, cache, (n_out + out_per_group - 1) / out_per_group, s, job, x, nb, rin);
 }
 
 template <int PASSES, int WPR, bool PAIR, bool MULTI, int NORM, bool XW = false>
 int launch_staged(const Q6Job& job, int64_t n_out, const uint16_t* x, int nb, const RmsIn& rin, hipStream_t s) {
     if constexpr (NORM == 0) {
+        if constexpr (!PAIR && WPR == 4 && PASSES <= 3) {
+            if (aligned(x, 16))  // 128-bit loads of x; a wave's own loads take any alignment
+                return launch_staged_vw<PASSES, WPR, PAIR, MULTI, NORM, XW, 0, true>(job, n_out, x, nb, rin, s);
+        }
         return launch_staged_vw<PASSES, WPR, PAIR, MULTI, NORM, XW, 0>(job, n_out, x, nb, rin, s);
     } else {
         constexpr int nw = staged_waves<WPR, PAIR, NORM>();
