@@ -430,7 +430,7 @@ constexpr int staged_waves() { return XL || (NORM && WPR == 1) ? 8 : (PAIR && WP
 // costs its loads, masks and reductions whether or not it is used).
 // CLOCK: the instrumented copy (FENCE_WAVE_CLOCK builds launch it on the grid
 // the plain kernel gets); every product launch has CLOCK = false.
-// XL (16-byte aligned x, rows on four waves of at most three passes): x comes
+// XL (16-byte aligned x, few rows on four waves of at most three passes): x comes
 // through LDS once per 8-wave workgroup.  A wave that loads its own x reads 2
 // KB a pass for 840 bytes of weights and visits one or two rows, so over the
 // six 4-wave workgroups of a CU x was more of its traffic than W.  Same bits.
@@ -1175,7 +1175,15 @@ template <int PASSES, int WPR, bool PAIR, bool MULTI, int NORM, bool XW = false>
 int launch_staged(const Q6Job& job, int64_t n_out, const uint16_t* x, int nb, const RmsIn& rin, hipStream_t s) {
     if constexpr (NORM == 0) {
         if constexpr (!PAIR && WPR == 4 && PASSES <= 3) {
-            if (aligned(x, 16))  // 128-bit loads of x; a wave's own loads take any alignment
+            // 128-bit loads of x; a wave's own loads take any alignment.  Past two
+            // (one-pass rows) or three (three-pass rows) rounds of the 1536 rows
+            // resident at once, a wave's own x serves more rows and the wider
+            // workgroup's barriers cost more than it saves.  GPU time without
+            // -> with: 14 blocks, 1536 rows 3.81 -> 3.75 us, 2560 4.44 -> 4.46,
+            // 4096 5.51 -> 5.63, 5120 6.40 -> 6.54; 33 blocks, 1536 rows 6.64 ->
+            // 6.16, 4096 10.63 -> 10.47, 5120 12.69 -> 12.80.
+            constexpr int64_t kSharedXRows = PASSES == 1 ? 3072 : 4608;
+            if (aligned(x, 16) && n_out <= kSharedXRows)
                 return launch_staged_vw<PASSES, WPR, PAIR, MULTI, NORM, XW, 0, true>(job, n_out, x, nb, rin, s);
         }
         return launch_staged_vw<PASSES, WPR, PAIR, MULTI, NORM, XW, 0>(job, n_out, x, nb, rin, s);

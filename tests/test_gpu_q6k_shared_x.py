@@ -21,7 +21,7 @@ def blocks(rng, rows, nb):
 
 
 @pytest.mark.parametrize("nb", [13, 16, 33, 38, 48, 49, 64])
-@pytest.mark.parametrize("rows", [8, 24, 3 * 8 * 257])
+@pytest.mark.parametrize("rows", [8, 24, 3072, 4608, 3 * 8 * 257])  # the largest that share x, and more
 def test_x_alignment_does_not_change_the_bits(nb, rows):
     rng = np.random.default_rng(nb * 1000 + rows)
     x = rng.standard_normal(256 * nb).astype(np.float16)
