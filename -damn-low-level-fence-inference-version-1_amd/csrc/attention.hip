@@ -255,10 +255,10 @@ __device__ __forceinline__ void write_head_half(float* out, uint16_t* out16, int
 // 16 workgroups) the launch is ~1.6 us, q arrives 1.2 us after a workgroup
 // starts on an idle CU and up to 3.8 us after on one whose earlier workgroups
 // already asked for their rows, scores to outputs take ~1 us, the partials'
-// stores, the arrival and the merge ~2 us.  V's loads behind q's arrival and
-// the row sums in registers instead of LDS took the call from 8.01 to 7.63 us
-// (GPU time, Qwen3-4B's 32 x 8 heads); K behind q too: 8.3 us, four heads per
-// workgroup: 9.8 us.
+// stores, the arrival and the merge ~2 us.  V's loads behind q's arrival took
+// the call from 8.45 to 8.26 us (launches back to back, caches of 40 layers in
+// turn, Qwen3-4B's 32 x 8 heads); K behind q too: +0.7 us, four heads per
+// workgroup: +2.2 us.
 // ARRIVE (with !FINAL, at most kWave splits): no merge launch.  The partials
 // are written with device-coherent stores (agent-scope atomic stores, which
 // write through the XCD's L2); once they have completed, the workgroup bumps
@@ -286,8 +286,7 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(float* __restrict_
     static_assert(!QK || (kThreads >= 3 * kWave && kUnits <= 2 * kWave), "prologue lanes");
     static_assert(kSub == kWave, "one position of a sub-chunk per lane in (B)");
     __shared__ float sp[2][GT][kSub];      // scores of even / odd sub-chunks
-    constexpr int kWaves = kThreads / kWave;
-    __shared__ float xo[kWaves][GT][HD];   // each wave's sums of its position groups
+    __shared__ __align__(16) float xo[kPG][GT][HD];
     __shared__ __align__(16) float qcs[QK ? HD : 1];            // prologue: cos[HALF] then sin[HALF]
     __shared__ __align__(16) float qs[QK ? GT : 1][HD];         // prologue: the prepared q heads
     __shared__ __align__(16) uint16_t kvn[QK ? 2 : 1][HD];      // prologue: position pos's k, v (binary16)
@@ -573,23 +572,25 @@ __global__ __launch_bounds__(kThreads) void attn_split_kernel(float* __restrict_
         }
     }
 
-    // Sum the position groups' outputs (they share the running maximum): the
-    // wave's four in registers, row r ending with dims 8 sl + 4 k + r, then
-    // the waves' through LDS.
+    // Sum the position groups' outputs (they share the running maximum), in
+    // group order from 0: the order is part of the result.  (The wave's four
+    // groups by row swaps first, then four waves: another rounding of most
+    // elements, which the binary16 output carries into every later layer.)
 #pragma unroll
-    for (int g = 0; g < GT; ++g)
-#pragma unroll
-        for (int k = 0; k < 2; ++k)
-            xo[wave][g][8 * sl + 4 * k + (lane >> 4)] =
-                row_sums4(o[g][4 * k], o[g][4 * k + 1], o[g][4 * k + 2], o[g][4 * k + 3]);
+    for (int g = 0; g < GT; ++g) {
+        f4 lo, hi;
+        lo.x = o[g][0], lo.y = o[g][1], lo.z = o[g][2], lo.w = o[g][3];
+        hi.x = o[g][4], hi.y = o[g][5], hi.z = o[g][6], hi.w = o[g][7];
+        *reinterpret_cast<f4*>(&xo[pg][g][8 * sl]) = lo;
+        *reinterpret_cast<f4*>(&xo[pg][g][8 * sl + 4]) = hi;
+    }
     __syncthreads();
     // thread (g, d): one output element of one head
     for (int e = threadIdx.x; e < GT * HD; e += kThreads) {
         const int g = e / HD, d = e % HD;
         if (g >= ng) continue;
-        float acc = xo[0][g][d];
-#pragma unroll
-        for (int k = 1; k < kWaves; ++k) acc += xo[k][g][d];
+        float acc = 0.0f;
+        for (int k = 0; k < kPG; ++k) acc += xo[k][g][d];
         float l = hl[0], mg = hm[0];
 #pragma unroll
         for (int k = 1; k < GT; ++k) {
