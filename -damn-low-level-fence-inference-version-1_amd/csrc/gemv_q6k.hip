@@ -430,14 +430,16 @@ constexpr int staged_waves() { return XL || (NORM && WPR == 1) ? 8 : (PAIR && WP
 // costs its loads, masks and reductions whether or not it is used).
 // CLOCK: the instrumented copy (FENCE_WAVE_CLOCK builds launch it on the grid
 // the plain kernel gets); every product launch has CLOCK = false.
-// XL (16-byte aligned x, few rows on four waves of at most three passes): x comes
-// through LDS once per 8-wave workgroup.  A wave that loads its own x reads 2
-// KB a pass for 840 bytes of weights and visits one or two rows, so over the
-// six 4-wave workgroups of a CU x was more of its traffic than W.  Same bits.
-// Measured, GPU time: down 2560 x 9728 7.88 -> 7.44 us, o 2560 x 4096 4.39 ->
-// 4.32; with four passes (rows of 49-64 blocks) x takes 32 KB and only 16
-// waves fit a CU instead of 24: 4096 x 14336 13.3 -> 13.7, so those keep a
-// wave's own loads.
+// XL (16-byte aligned x, three-pass rows on four waves; which launches:
+// shares_x): x comes through LDS once per 8-wave workgroup of two rows.  A
+// wave that loads its own x reads 2 KB a pass for 840 bytes of weights and
+// visits one or two rows, so over the six 4-wave workgroups of a CU x was more
+// of its traffic than W.  Same bits.  Measured, GPU time: down 2560 x 9728
+// 8.03 -> 7.72 us.  The other layouts keep a wave's own loads: rows of 13-16
+// blocks (XW) read x once for as many bytes of W and lose more to the wider
+// workgroups (o 2560 x 4096 4.39 us, 4.43 with XL; 4096 x 4096 5.45, 5.56);
+// with four passes (49-64 blocks) x takes 32 KB and only 16 waves fit a CU
+// instead of 24: 4096 x 14336 13.3, 13.7.
 template <int PASSES, int WPR, bool PAIR, bool MULTI, int NORM, bool XW = false, bool CLOCK = false, int VW = 0,
           bool XL = false>
 __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM, XL>())) void gemv_q6k_staged_kernel(
@@ -446,7 +448,7 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM, XL>())) void
     // prefetch the next row group: XW launches, and where the switches below ask
     constexpr bool PF = XW || (FENCE_GEMV_Q6K_PF_NORM && NORM != 0 && WPR == 1 && !PAIR) ||
                         (FENCE_GEMV_Q6K_PF_SPLIT && NORM == 0 && WPR > 1 && !PAIR);
-    static_assert(!XL || (NORM == 0 && !PAIR && WPR == 4 && PASSES <= 3), "XL: plain rows of four waves");
+    static_assert(!XL || (NORM == 0 && !PAIR && !XW && WPR == 4 && PASSES == 3), "XL: plain rows of four waves");
     constexpr int NW = staged_waves<WPR, PAIR, NORM, XL>();
     constexpr int kSegBytes = 4 * PASSES * kBlockBytes + 32;  // + alignment slack
     constexpr int kBufBytes = (kSegBytes + 15) / 16 * 16;
@@ -1123,28 +1125,42 @@ __global__ __launch_bounds__(kThreads) void gemv_q6k_direct_kernel(const Q6Job j
     }
 }
 
-// A resident grid of `threads`-lane workgroups for `occ_kernel`: CUs x its
-// occupancy per CU (cached per device in `cache`), at most `groups`; launches
-// `kernel` on it (the same kernel, or its instrumented copy).
-template <class OccKernel, class Kernel, class... Args>
-int launch_grid_as(OccKernel occ_kernel, Kernel kernel, int threads, std::atomic<int>* cache, int64_t groups,
-                   hipStream_t s, const Args&... args) {
+// The current device's CUs, and how many `threads`-lane workgroups of `kernel`
+// it holds at once (cached per device in `cache`).
+template <class Kernel>
+int resident_grid(Kernel kernel, int threads, std::atomic<int>* cache, int* cus, int* grid) {
+    static std::atomic<int> cu_cache[64];
     int dev = 0;
     if (hipError_t e = hipGetDevice(&dev); e != hipSuccess) return hip_status(e);
     if (dev < 0 || dev >= 64) return FENCE_ERROR_INVALID_VALUE;
+    int n = cu_cache[dev].load(std::memory_order_relaxed);
+    if (n == 0) {
+        if (hipError_t e = hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev); e != hipSuccess)
+            return hip_status(e);
+        cu_cache[dev].store(n, std::memory_order_relaxed);
+    }
     int g = cache[dev].load(std::memory_order_relaxed);
     if (g == 0) {
-        int cus = 0, per_cu = 0;
-        if (hipError_t e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev); e != hipSuccess)
-            return hip_status(e);
-        if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, occ_kernel, threads, 0);
-            e != hipSuccess)
+        int per_cu = 0;
+        if (hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, threads, 0); e != hipSuccess)
             return hip_status(e);
         const int cap = FENCE_GEMV_Q6K_WG_PER_CU * 4 * kWave / threads;  // in waves: of 4-wave workgroups
         if (FENCE_GEMV_Q6K_WG_PER_CU > 0 && per_cu > cap) per_cu = cap;
-        g = cus * (per_cu > 0 ? per_cu : 1);
+        g = n * (per_cu > 0 ? per_cu : 1);
         cache[dev].store(g, std::memory_order_relaxed);
     }
+    *cus = n;
+    *grid = g;
+    return FENCE_SUCCESS;
+}
+
+// Launches `kernel` (`occ_kernel`, or its instrumented copy) on a resident
+// grid of `threads`-lane workgroups, at most `groups` of them.
+template <class OccKernel, class Kernel, class... Args>
+int launch_grid_as(OccKernel occ_kernel, Kernel kernel, int threads, std::atomic<int>* cache, int64_t groups,
+                   hipStream_t s, const Args&... args) {
+    int cus = 0, g = 0;
+    if (int st = resident_grid(occ_kernel, threads, cache, &cus, &g)) return st;
     if (!FENCE_GEMV_Q6K_RESIDENT) g = 0x7fffffff;
     int64_t w = groups < g ? groups : g;
     if (FENCE_GEMV_Q6K_BALANCED && w > 0) {
@@ -1171,19 +1187,37 @@ int launch_staged_vw(const Q6Job& job, int64_t n_out, const uint16_t* x, int nb,
                           kWave * nw, cache, (n_out + out_per_group - 1) / out_per_group, s, job, x, nb, rin);
 }
 
+// Whether n_out three-pass rows share x (XL) on `cus` CUs that hold `resident`
+// two-row workgroups at once: up to three rounds of them (past that a wave's
+// own x serves enough rows), and not where handing rows out in pairs leaves
+// some CUs a row more than one at a time would, unless the rounds before the
+// last have already earned that row: half the CUs' worth of extra workgroups
+// costs what sharing x saves in a round or two.  Measured, 33 / 48 blocks, GPU
+// time without -> with on 256 CUs x 3 workgroups: even, 512 rows 4.01 -> 3.93
+// / 4.12 -> 4.05 us, 1536 6.55 -> 5.99 / 6.86 -> 6.28, 4608 11.85 -> 11.66 /
+// 12.83 -> 12.11; uneven and earned, 1792 6.75 -> 6.57 / 7.24 -> 6.91, 3840
+// 10.11 -> 10.01 / 11.07 -> 10.38; uneven, 256 3.40 -> 3.77 / 3.47 -> 3.81, 768
+// 4.69 -> 4.94 / 4.83 -> 5.09, 2816 8.69 -> 8.93 / 9.23 -> 9.27, 4352 11.02 ->
+// 11.57 / 11.57 -> 11.96; past three rounds, 5888 13.47 -> 14.33 / 14.19 ->
+// 15.06.
+constexpr bool shares_x(int64_t n_out, int64_t cus, int64_t resident) {
+    const int64_t groups = (n_out + 1) / 2;
+    const int64_t full = groups / resident, last = groups % resident;
+    const bool even = 2 * ((groups + cus - 1) / cus) <= (n_out + cus - 1) / cus;
+    return groups <= 3 * resident && (even || 2 * last <= cus * (2 * full - 1));
+}
+
 template <int PASSES, int WPR, bool PAIR, bool MULTI, int NORM, bool XW = false>
 int launch_staged(const Q6Job& job, int64_t n_out, const uint16_t* x, int nb, const RmsIn& rin, hipStream_t s) {
     if constexpr (NORM == 0) {
-        if constexpr (!PAIR && WPR == 4 && PASSES <= 3) {
-            // 128-bit loads of x; a wave's own loads take any alignment.  Past two
-            // (one-pass rows) or three (three-pass rows) rounds of the 1536 rows
-            // resident at once, a wave's own x serves more rows and the wider
-            // workgroup's barriers cost more than it saves.  GPU time without
-            // -> with: 14 blocks, 1536 rows 3.81 -> 3.75 us, 2560 4.44 -> 4.46,
-            // 4096 5.51 -> 5.63, 5120 6.40 -> 6.54; 33 blocks, 1536 rows 6.64 ->
-            // 6.16, 4096 10.63 -> 10.47, 5120 12.69 -> 12.80.
-            constexpr int64_t kSharedXRows = PASSES == 1 ? 3072 : 4608;
-            if (aligned(x, 16) && n_out <= kSharedXRows)
+        if constexpr (!PAIR && WPR == 4 && PASSES == 3) {
+            static std::atomic<int> cache[64];
+            int cus = 0, resident = 0;
+            if (int st = resident_grid(gemv_q6k_staged_kernel<PASSES, WPR, PAIR, MULTI, NORM, XW, false, 0, true>,
+                                       kWave * staged_waves<WPR, PAIR, NORM, true>(), cache, &cus, &resident))
+                return st;
+            // 128-bit loads of x; a wave's own loads take any alignment
+            if (aligned(x, 16) && shares_x(n_out, cus, resident))
                 return launch_staged_vw<PASSES, WPR, PAIR, MULTI, NORM, XW, 0, true>(job, n_out, x, nb, rin, s);
         }
         return launch_staged_vw<PASSES, WPR, PAIR, MULTI, NORM, XW, 0>(job, n_out, x, nb, rin, s);
