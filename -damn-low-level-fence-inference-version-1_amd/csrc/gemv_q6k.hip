@@ -55,15 +55,20 @@
 // interleaved runs each): 1,852 and 1,854 us per token with 1 against 1,768
 // and 1,767 with 0 -- wave lifetimes vary by several us within a launch
 // whatever the group count, so fewer workgroups only lose parallelism.
-// Most workgroups per CU in a resident grid (0: as many as fit).  6 trims
-// the 4-wave launches (down: 7 fit, o: 8) and leaves the 8-wave ones (2
-// fit); decode steps ran ~10 us per token faster than with every resident
-// workgroup, and slower with 5 (+15-20 us) or level with 4.
-#ifndef FENCE_GEMV_Q6K_WG_PER_CU
-#define FENCE_GEMV_Q6K_WG_PER_CU 6
-#endif
 #ifndef FENCE_GEMV_Q6K_BALANCED
 #define FENCE_GEMV_Q6K_BALANCED 0
+#endif
+// Most waves per CU in a resident grid, counted in 4-wave workgroups (0: as
+// many as fit): 6 is 24 waves, six 4-wave or three 8-wave workgroups.  It
+// trims the 4-wave launches of few registers (o: 8 fit) and the 8-wave ones
+// of at most four blocks a row (4 fit); the other 8-wave launches hold two or
+// three by themselves.  Decode steps ran ~10 us per token faster than with
+// every resident workgroup, and slower with 5 (+15-20 us) or level with 4.
+// Three 8-wave workgroups against the four that fit, rows of four blocks, GPU
+// time: q/k/v 8192 rows 4.50 against 4.80 us, 16384 6.28 against 6.64, gate/up
+// 9728 6.95 against 7.24; at most 6144 rows level.
+#ifndef FENCE_GEMV_Q6K_WG_PER_CU
+#define FENCE_GEMV_Q6K_WG_PER_CU 6
 #endif
 // 1: rows of 33-40 blocks take two waves of up to five passes (20 block
 // slots for 17-20 blocks) instead of four waves of three passes (12 slots for
@@ -121,9 +126,12 @@ static_assert(FENCE_GEMV_Q6K_PAIRW == 0 || FENCE_GEMV_Q6K_PAIRW == 4 || FENCE_GE
 // computed (as XW launches do) in the one-wave launches with the RMSNorm
 // prologue (q/k/v) -- PF_NORM -- and in launches of several waves per row
 // (down) -- PF_SPLIT; 0: each group after the previous one.  Same results.
-// PF_NORM: q/k/v of Qwen3-4B (6144 x 2560) 6.65 us without, 6.28 with, GPU
-// time (two 8-wave workgroups per CU either way, half of which take a second
-// group).  PF_SPLIT: decode steps within the spread of the runs.
+// PF_NORM, GPU time without -> with: where waves take a second group, q/k/v
+// of Qwen3-4B (6144 rows of 10 blocks) 6.64 -> 6.20 us, 9216 rows of 5 blocks
+// 6.40 -> 6.01; where every wave has one group its registers and branch cost
+// up to 0.1 us (1024 rows of 10 blocks 4.18 -> 4.31), and at 16 blocks it
+// costs that much or more (4096 rows 6.68 -> 6.97).  PF_SPLIT: decode steps
+// within the spread of the runs.
 #ifndef FENCE_GEMV_Q6K_PF_NORM
 #define FENCE_GEMV_Q6K_PF_NORM 1
 #endif
@@ -412,8 +420,8 @@ constexpr int staged_waves() { return XL || (NORM && WPR == 1) ? 8 : (PAIR && WP
 // <= 16 blocks.  LDS: one buffer of kSegBytes per wave + red[].  A workgroup
 // of NW waves takes NW / WPR rows per group; with PAIR the first half of them
 // are gate rows and the second half the same rows of up.  NORM: x from
-// `rin` (see RmsIn), staged through the same LDS before the first group's
-// blocks are; NORM (1 or 2) is the norm kernel's float4s per lane, rin.vpt.
+// `rin` (see RmsIn), in LDS of its own behind the wave buffers; NORM (1 or 2)
+// is the norm kernel's float4s per lane, rin.vpt.
 // XW (PASSES * WPR = 4, rows of 13-16 blocks): the one-wave layout <4, 1>
 // spread over WPR waves -- wave s takes passes PASSES*s .. PASSES*s +
 // PASSES - 1 (blocks from 4 * PASSES * s on), and each pass's lane values go
@@ -423,8 +431,9 @@ constexpr int staged_waves() { return XL || (NORM && WPR == 1) ? 8 : (PAIR && WP
 // XW launches also load each wave's next row group while the current one is
 // computed (one chunk slot per lane: 4 VGPRs).  Measured on MI355X, p50 of
 // 400, in-process A/B: the o projection 2560 x 4096 4.92 -> 4.60 us, Llama-3-8B
-// 4096 x 4096 6.44 -> 5.80 us; the same prefetch in the other layouts cost
-// more registers than it saved (gate/up pair, 9728 x 2560) or changed nothing.
+// 4096 x 4096 6.44 -> 5.80 us.  The one-wave NORM rows prefetch too
+// (FENCE_GEMV_Q6K_PF_NORM above); in the staged gate/up pair (9728 x 2560) it
+// cost more registers than it saved, in the other layouts it changed nothing.
 // VW (NORM launches): the norm's 64-lane virtual waves each wave holds,
 // ceil((T / 64) / NW), chosen at launch so no slot is always empty (a slot
 // costs its loads, masks and reductions whether or not it is used).
@@ -578,7 +587,11 @@ __global__ __launch_bounds__((kWave * staged_waves<WPR, PAIR, NORM, XL>())) void
         // workgroup by 1-2 us, and nothing starts without it.  With the wave
         // sums read at once (fold_waves) and the prefetch above, q/k/v of
         // Qwen3-4B went from 7.0 to 6.3 us: 0.2 the order, 0.1 the barrier
-        // and the sums, 0.4 the prefetch.
+        // and the sums, 0.4 the prefetch.  A launch of at most one workgroup
+        // per CU has no second one and keeps the order: GPU time asked for
+        // before -> after the row at 1024 rows, 4 blocks 3.33 -> 3.22 us, 8
+        // 3.77 -> 3.60, 10 4.31 -> 4.31, 12 4.35 -> 4.35, 16 4.97 -> 4.74, 32
+        // 7.43 -> 7.10 (12 blocks, 2048 rows: 4.52 -> 4.61).
         // h = hid (+ res), zero past the row; workgroup 0 stores it; then
         // each slot keeps only w * h, the first product of the norm's output
         const int nvw = rin.T / kWave;
@@ -833,7 +846,7 @@ __global__ __launch_bounds__(kWave * NW) __attribute__((amdgpu_waves_per_eu(FENC
     uint32_t xh[PASSES][8];
     float kb[PASSES][4];
     // MERGE: x of the merged pass's block, 4 (PASSES - 1) + (bslot & 1), for
-    // every slot (the last pass of xh masks slots 2, 3)
+    // every slot (in the last pass of xh slots 2, 3 hold a clamped block's)
     uint32_t xm[1][8];
     float km[1][4];
     const int b0m = 4 * (PASSES - 1) + (bslot & 1) - bslot;
